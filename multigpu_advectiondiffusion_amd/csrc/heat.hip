@@ -935,9 +935,10 @@ extern "C" int mgad_heat7_fe_steps(hipStream_t stream, unsigned int nx, unsigned
         set_error(MGAD_ERR_INVALID_ARG);
         return MGAD_ERR_INVALID_ARG;
     }
+    if (!use_graph || stream == nullptr) return enqueue_heat(stream, nx, ny, nz, kx, ky, kz, dt, u, w, nsteps);
+    std::lock_guard<std::recursive_mutex> lock(host_mutex());
     // a graph of the whole call where it takes about 48 launches or more
-    if (!use_graph || stream == nullptr || nsteps < 48 * 4)
-        return enqueue_heat(stream, nx, ny, nz, kx, ky, kz, dt, u, w, nsteps);
+    if (nsteps < 48 * 4) return enqueue_heat(stream, nx, ny, nz, kx, ky, kz, dt, u, w, nsteps);
     static std::map<HeatKey, hipGraphExec_t> cache;
     const HeatKey key{stream, nx, ny, nz, kx, ky, kz, dt, u, w, nsteps};
     return replay_steps(cache, 16, key, stream, 1, 1,
@@ -956,6 +957,9 @@ extern "C" int mgad_heat13_rk3_steps(hipStream_t stream, unsigned int nx, unsign
     }
     if (nsteps == 0) return MGAD_OK;
     const DiffCoef c = diff_coef();
+    std::unique_lock<std::recursive_mutex> lock(host_mutex(), std::defer_lock);
+    const bool graph = use_graph && stream != nullptr;
+    if (graph) lock.lock();
     // a step goes u -> w1 or w1 -> u; an odd count's last one is copied back
     const int pairs = nsteps / 2;
     int st = MGAD_OK;
@@ -963,7 +967,7 @@ extern "C" int mgad_heat13_rk3_steps(hipStream_t stream, unsigned int nx, unsign
         const int r = enqueue_heat13(stream, nx, ny, nz, c, dt, u, w1);
         return r ? r : enqueue_heat13(stream, nx, ny, nz, c, dt, w1, u);
     };
-    if (!use_graph || stream == nullptr) {
+    if (!graph) {
         for (int s = 0; s < pairs && !st; s++) st = pair();
     } else {
         using Key = std::tuple<hipStream_t, unsigned, unsigned, unsigned, double, double, double, double, double *,

@@ -1,0 +1,54 @@
+"""The host side of the step calls on a HIP runtime that runs nothing and
+writes down what it is asked for (tests/fake_hip): what is launched, captured,
+replayed and waited for.  No GPU and no GPU code: the results of captured and
+of direct steps are compared on the device by test_gpu_graph_lengths.py."""
+import json
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="no host compiler")
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-pthread", "-D__HIP_PLATFORM_AMD__",
+                    f"-I{ROCM}/include", os.path.join(HERE, "fake_hip", "fake_hip.cpp"), "-o", lib], check=True)
+
+    def go(script):
+        r = subprocess.run([sys.executable, os.path.join(HERE, "fake_hip", "launches.py"), lib], input=script,
+                           capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stderr[-4000:]
+        return json.loads(r.stdout)
+
+    return go
+
+
+# a call long enough to be captured
+LONG = {"periodic": 20, "slab": 20, "reference": 20, "weno7": 20, "heat13": 101, "heat7": 203}
+
+
+@pytest.mark.parametrize("kind", LONG)
+def test_short_call_waits_for_another_threads_capture(run, kind):
+    """Two host threads on one stream: steps that one launches must not be
+    recorded into the graph that the other captures."""
+    log = run(f"""
+fake.fake_hold_captures(400)
+t = threading.Thread(target=call, args=({kind!r}, {LONG[kind]}))
+t.start()
+while not fake.fake_captures_open() and t.is_alive():
+    time.sleep(0.001)
+opened = fake.fake_captures_open()
+rc = call({kind!r}, 3)
+t.join()
+out = [opened, rc, log()]
+""")
+    assert log[:2] == [1, 0] and "n" in log[2]
+    assert "x" not in log[2]

@@ -431,14 +431,17 @@ int mgad_batch_init(hipStream_t stream, int precision,
                     double tend, double cfl, mgad_batch *out);
 
 /* nsteps SSP-RK3 steps of every problem: three persistent launches per step
- * (each walks the whole work list); use_graph replays a hipGraph
- * of 16 steps, and the rest is launched directly.  Each problem keeps its own dt and LF alpha, and
- * its results are bit-identical to advancing it alone. */
+ * (each walks the whole work list).  With use_graph the steps are replays of a
+ * hipGraph of 16 steps, the rest launched directly, and the call returns when
+ * they have ended (it synchronises the stream); without, it is asynchronous on
+ * stream.  Each problem keeps its own dt and LF alpha, and its results are
+ * bit-identical to advancing it alone. */
 int mgad_batch_steps(hipStream_t stream, const mgad_batch *batch, int nsteps,
                      int use_graph);
 
 /* The same steps with the single-problem kernel launched problem by problem
- * (3 launches per problem per step, each with its tuned configuration). */
+ * (3 launches per problem per step, each with its tuned configuration);
+ * use_graph as for mgad_batch_steps. */
 int mgad_batch_steps_serial(hipStream_t stream, const mgad_batch *batch,
                             const mgad_problem *probs, int nsteps,
                             int use_graph);

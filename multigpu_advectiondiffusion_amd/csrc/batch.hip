@@ -380,13 +380,14 @@ int enqueue_serial_step(hipStream_t stream, const mgad_batch &b, const mgad_prob
 
 // nsteps times `enqueue` (a step of `launches` launches): replays of a graph of
 // graph_steps(launches) steps, captured for the call, and the rest (or a short
-// call) directly.
+// call) directly.  With use_graph the call returns when the steps have ended.
 template <class F>
 int run_graph(hipStream_t stream, int nsteps, int use_graph, int launches, F &&enqueue) {
+    const bool graph = use_graph && stream != nullptr;
     const int per = graph_steps(launches);
     int st = MGAD_OK, done = 0;
-    if (use_graph && stream != nullptr && nsteps >= per) {
-        hipGraphExec_t exec = nullptr;
+    hipGraphExec_t exec = nullptr;
+    if (graph && nsteps >= per) {
         st = capture_graph(stream, &exec, [&] {
             int r = MGAD_OK;
             for (int s = 0; s < per && !r; s++) r = enqueue();
@@ -394,11 +395,13 @@ int run_graph(hipStream_t stream, int nsteps, int use_graph, int launches, F &&e
         });
         if (st) return st;
         for (; done + per <= nsteps && !st; done += per) st = check_hip(hipGraphLaunch(exec, stream));
-        const int sst = check_hip(hipStreamSynchronize(stream));
-        (void)hipGraphExecDestroy(exec);
-        if (!st) st = sst;
     }
     for (; done < nsteps && !st; done++) st = enqueue();
+    if (graph) {
+        const int sst = check_hip(hipStreamSynchronize(stream));
+        if (exec) (void)hipGraphExecDestroy(exec);
+        if (!st) st = sst;
+    }
     return st;
 }
 

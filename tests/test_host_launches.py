@@ -52,3 +52,16 @@ out = [opened, rc, log()]
 """)
     assert log[:2] == [1, 0] and "n" in log[2]
     assert "x" not in log[2]
+
+
+@pytest.mark.parametrize("n", [0, 3, 16, 18])
+@pytest.mark.parametrize("kind", ["batch", "serial"])
+def test_batch_calls_with_a_graph_return_when_the_steps_have_ended(run, kind, n):
+    with_graph, without = run(f"""
+assert call({kind!r}, {n}) == 0
+a = log()
+assert call({kind!r}, {n}, graph=0) == 0
+out = [a, log()]
+""")
+    assert with_graph.endswith("W")
+    assert "W" not in without

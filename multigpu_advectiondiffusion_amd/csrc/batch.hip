@@ -385,7 +385,8 @@ template <class F>
 int run_graph(hipStream_t stream, int nsteps, int use_graph, int launches, F &&enqueue) {
     const bool graph = use_graph && stream != nullptr;
     const int per = graph_steps(launches);
-    int st = MGAD_OK, done = 0;
+    int st = graph ? refuse_capture(stream) : MGAD_OK, done = 0;
+    if (st) return st;
     hipGraphExec_t exec = nullptr;
     if (graph && nsteps >= per) {
         st = capture_graph(stream, &exec, [&] {

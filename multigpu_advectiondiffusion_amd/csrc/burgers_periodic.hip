@@ -552,6 +552,7 @@ int run_steps(int precision, hipStream_t stream, const mgad_scheme *scheme, unsi
         return MGAD_OK;
     }
     std::lock_guard<std::recursive_mutex> lock(host_mutex());
+    if (const int st = refuse_capture(stream)) return st;
     const LaunchCfg cfg = launch_cfg(precision, *scheme, nx, ny, nz);
     const GraphKey key{stream, precision, scheme->weno, scheme->p, scheme->eps, nx, ny, nz, dx, dy, dz,
                        u,      w1,        w2,           ctrl,       cfg.tile,  cfg.kchunk};

@@ -440,6 +440,9 @@ extern "C" int mgad_burgers_ref_steps(hipStream_t stream, const mgad_scheme *sch
     }
     if (nsteps == 0) return MGAD_OK;
     std::lock_guard<std::recursive_mutex> lock(host_mutex());
+    if (use_graph && stream != nullptr) {
+        if (const int st = refuse_capture(stream)) return st;
+    }
     RefLaunch L = ref_launch(*scheme, viscous != 0, nx, ny, nz, dx, dy, dz);
     L.g.amax = ref_amax_slots(stream);
     if (!L.g.amax) return MGAD_ERR_HIP;

@@ -935,8 +935,10 @@ extern "C" int mgad_heat7_fe_steps(hipStream_t stream, unsigned int nx, unsigned
         set_error(MGAD_ERR_INVALID_ARG);
         return MGAD_ERR_INVALID_ARG;
     }
-    if (!use_graph || stream == nullptr) return enqueue_heat(stream, nx, ny, nz, kx, ky, kz, dt, u, w, nsteps);
+    if (!use_graph || stream == nullptr || nsteps == 0)
+        return enqueue_heat(stream, nx, ny, nz, kx, ky, kz, dt, u, w, nsteps);
     std::lock_guard<std::recursive_mutex> lock(host_mutex());
+    if (const int st = refuse_capture(stream)) return st;
     // a graph of the whole call where it takes about 48 launches or more
     if (nsteps < 48 * 4) return enqueue_heat(stream, nx, ny, nz, kx, ky, kz, dt, u, w, nsteps);
     static std::map<HeatKey, hipGraphExec_t> cache;
@@ -959,7 +961,10 @@ extern "C" int mgad_heat13_rk3_steps(hipStream_t stream, unsigned int nx, unsign
     const DiffCoef c = diff_coef();
     std::unique_lock<std::recursive_mutex> lock(host_mutex(), std::defer_lock);
     const bool graph = use_graph && stream != nullptr;
-    if (graph) lock.lock();
+    if (graph) {
+        lock.lock();
+        if (const int st = refuse_capture(stream)) return st;
+    }
     // a step goes u -> w1 or w1 -> u; an odd count's last one is copied back
     const int pairs = nsteps / 2;
     int st = MGAD_OK;

@@ -65,3 +65,20 @@ out = [a, log()]
 """)
     assert with_graph.endswith("W")
     assert "W" not in without
+
+
+@pytest.mark.parametrize("kind", [*LONG, "batch", "serial"])
+def test_graph_calls_are_refused_while_the_caller_captures(run, kind):
+    """Whatever their length, and without a trace in the caller's capture;
+    without a graph the same steps are recorded into it."""
+    out = run(f"""
+def under_capture(n, graph):
+    g = ctypes.c_void_p()
+    fake.hipStreamBeginCapture(0x77, 0)
+    rc = call({kind!r}, n, graph)
+    fake.hipStreamEndCapture(0x77, ctypes.byref(g))
+    return rc, log()
+out = [under_capture(2, 1), under_capture(250, 1), under_capture(2, 0)]
+""")
+    assert out[0] == [3, "[]"] and out[1] == [3, "[]"]  # MGAD_ERR_HIP
+    assert out[2][0] == 0 and "n" in out[2][1]

@@ -378,32 +378,23 @@ int enqueue_serial_step(hipStream_t stream, const mgad_batch &b, const mgad_prob
     return MGAD_OK;
 }
 
-// nsteps times `enqueue` (a step of `launches` launches): replays of a graph of
-// graph_steps(launches) steps, captured for the call, and the rest (or a short
-// call) directly.  With use_graph the call returns when the steps have ended.
+// nsteps times `enqueue` (a step of `launches` launches): with use_graph partly
+// as replays of a graph captured for the call (graphed_steps), and the call
+// returns when the steps have ended.
 template <class F>
 int run_graph(hipStream_t stream, int nsteps, int use_graph, int launches, F &&enqueue) {
-    const bool graph = use_graph && stream != nullptr;
-    const int per = graph_steps(launches);
-    int st = graph ? refuse_capture(stream) : MGAD_OK, done = 0;
+    if (!use_graph || stream == nullptr) {
+        int st = MGAD_OK;
+        for (int s = 0; s < nsteps && !st; s++) st = enqueue();
+        return st;
+    }
+    int st = refuse_capture(stream);
     if (st) return st;
     hipGraphExec_t exec = nullptr;
-    if (graph && nsteps >= per) {
-        st = capture_graph(stream, &exec, [&] {
-            int r = MGAD_OK;
-            for (int s = 0; s < per && !r; s++) r = enqueue();
-            return r;
-        });
-        if (st) return st;
-        for (; done + per <= nsteps && !st; done += per) st = check_hip(hipGraphLaunch(exec, stream));
-    }
-    for (; done < nsteps && !st; done++) st = enqueue();
-    if (graph) {
-        const int sst = check_hip(hipStreamSynchronize(stream));
-        if (exec) (void)hipGraphExecDestroy(exec);
-        if (!st) st = sst;
-    }
-    return st;
+    st = graphed_steps(stream, nsteps, graph_steps(launches), false, exec, enqueue);
+    const int sst = check_hip(hipStreamSynchronize(stream));
+    if (exec) (void)hipGraphExecDestroy(exec);
+    return st ? st : sst;
 }
 
 int init_ctrls(hipStream_t stream, int precision, int nprob, const mgad_problem *p, double t0, double tend,

@@ -82,3 +82,42 @@ out = [under_capture(2, 1), under_capture(250, 1), under_capture(2, 0)]
 """)
     assert out[0] == [3, "[]"] and out[1] == [3, "[]"]  # MGAD_ERR_HIP
     assert out[2][0] == 0 and "n" in out[2][1]
+
+
+# launches a step, steps a graph, launches before a call's first step
+SHAPE = {"periodic": (3, 16, 0), "slab": (3, 16, 0), "reference": (3, 16, 2), "weno7": (5, 9, 0),
+         "heat13": (1, 48, 0)}
+
+
+@pytest.mark.parametrize("kind", SHAPE)
+def test_first_long_call_launches_before_it_captures(run, kind):
+    """The device has work when the host captures; later calls replay, and so
+    does the first one once four graphs' worth of steps has been launched."""
+    per_step, per, pre = SHAPE[kind]
+    n, many = per + 4, 6 * per + 4
+    first, second, other = run(f"""
+assert call({kind!r}, {n}) == 0
+a = log()
+assert call({kind!r}, {n}) == 0
+b = log()
+assert call({kind!r}, {many}, u=0x800000) == 0
+out = [a, b, log()]
+""")
+    nodes = per * per_step
+    graph, replay, rest = "[" + "n" * nodes + "]", f"R{nodes};", "L" * (4 * per_step)
+    assert first == "L" * (pre + n * per_step) + graph
+    assert second == "L" * pre + replay + rest
+    assert other == "L" * (pre + 4 * nodes) + graph + 2 * replay + rest
+
+
+@pytest.mark.parametrize("kind,per_step", [("batch", 3), ("serial", 6)])
+def test_batch_call_captures_only_what_it_replays_itself(run, kind, per_step):
+    short, long, execs = run(f"""
+assert call({kind!r}, {192 // per_step}) == 0
+a = log()
+assert call({kind!r}, {96 * 4 // per_step + 1}) == 0
+out = [a, log(), fake.fake_live_execs()]
+""")
+    assert short == "L" * 192 + "W"
+    assert long == "L" * 192 + "[" + "n" * 48 + "]" + 4 * "R48;" + "L" * per_step + "W"
+    assert execs == 0

@@ -840,18 +840,23 @@ int enqueue_heat7(hipStream_t s, unsigned nx, unsigned ny, unsigned nz, double k
     return check_launch();
 }
 
-// nsteps steps as an even number of launches (u -> w -> u ...), as few as the
-// most steps a launch takes allow and as equal as possible; a single step is
-// copied back.  Most steps a launch: 4, or 5 where the tall tile is taken.  A
+// Most steps a launch takes: 4, or 5 where the tall tile is taken.  A
 // fifth step costs the tall tile little (us a step at 512^3 with 2, 3, 4, 5
 // steps a launch: 304, 188, 172, 185; with 1: 384) and saves launches that
 // would only make their number even; the low tile loses more of its rows to
 // the halo (64^3: 2.59, 2.47, 2.43, 2.88; with 1: 3.23).
-int enqueue_heat(hipStream_t s, unsigned nx, unsigned ny, unsigned nz, double kx, double ky,
-                 double kz, double dt, double *u, double *w, int nsteps) {
+int heat7_most_steps(unsigned nx, unsigned ny, unsigned nz) {
     bool tall;
     heat7_steps_grid(nx, ny, nz, 4, tall);
-    const int tmax = tall ? 5 : 4;
+    return tall ? 5 : 4;
+}
+
+// nsteps steps as an even number of launches (u -> w -> u ...), as few as the
+// most steps a launch takes allow and as equal as possible; a single step is
+// copied back.
+int enqueue_heat(hipStream_t s, unsigned nx, unsigned ny, unsigned nz, double kx, double ky,
+                 double kz, double dt, double *u, double *w, int nsteps) {
+    const int tmax = heat7_most_steps(nx, ny, nz);
     int launches = (nsteps + tmax - 1) / tmax;
     if (launches < nsteps) launches += launches & 1;
     for (int it = 0, done = 0; it < launches; it++) {
@@ -915,10 +920,9 @@ struct HeatKey {
     unsigned nx, ny, nz;
     double kx, ky, kz, dt;
     double *u, *w;
-    int nsteps;
     bool operator<(const HeatKey &o) const {
-        return std::tie(s, nx, ny, nz, kx, ky, kz, dt, u, w, nsteps) <
-               std::tie(o.s, o.nx, o.ny, o.nz, o.kx, o.ky, o.kz, o.dt, o.u, o.w, o.nsteps);
+        return std::tie(s, nx, ny, nz, kx, ky, kz, dt, u, w) <
+               std::tie(o.s, o.nx, o.ny, o.nz, o.kx, o.ky, o.kz, o.dt, o.u, o.w);
     }
 };
 
@@ -939,12 +943,23 @@ extern "C" int mgad_heat7_fe_steps(hipStream_t stream, unsigned int nx, unsigned
         return enqueue_heat(stream, nx, ny, nz, kx, ky, kz, dt, u, w, nsteps);
     std::lock_guard<std::recursive_mutex> lock(host_mutex());
     if (const int st = refuse_capture(stream)) return st;
-    // a graph of the whole call where it takes about 48 launches or more
-    if (nsteps < 48 * 4) return enqueue_heat(stream, nx, ny, nz, kx, ky, kz, dt, u, w, nsteps);
-    static std::map<HeatKey, hipGraphExec_t> cache;
-    const HeatKey key{stream, nx, ny, nz, kx, ky, kz, dt, u, w, nsteps};
-    return replay_steps(cache, 16, key, stream, 1, 1,
-                        [&] { return enqueue_heat(stream, nx, ny, nz, kx, ky, kz, dt, u, w, nsteps); });
+    // whole graphs of 24 pairs of full launches, u -> w -> u, and the rest as a
+    // call without a graph; where that would be less than two full launches it
+    // gets a graph's steps too (launches of one step take twice the time a step)
+    const int t = heat7_most_steps(nx, ny, nz), per = graph_steps(2), full = per * 2 * t;
+    int graphs = nsteps / full;
+    const int left = nsteps - graphs * full;
+    if (graphs > 0 && left > 0 && left < 2 * t) graphs--;
+    int st = MGAD_OK;
+    if (graphs > 0) {
+        static std::map<HeatKey, hipGraphExec_t> cache;
+        const HeatKey key{stream, nx, ny, nz, kx, ky, kz, dt, u, w};
+        st = replay_steps(cache, 16, key, stream, graphs * per, per, [&] {
+            const int r = enqueue_heat7(stream, nx, ny, nz, kx, ky, kz, dt, u, w, t);
+            return r ? r : enqueue_heat7(stream, nx, ny, nz, kx, ky, kz, dt, w, u, t);
+        });
+    }
+    return st ? st : enqueue_heat(stream, nx, ny, nz, kx, ky, kz, dt, u, w, nsteps - graphs * full);
 }
 
 // The reference's heat step fused (SingleGPU/Diffusion3d_baselineCode/

@@ -121,3 +121,21 @@ out = [a, log(), fake.fake_live_execs()]
     assert short == "L" * 192 + "W"
     assert long == "L" * 192 + "[" + "n" * 48 + "]" + 4 * "R48;" + "L" * per_step + "W"
     assert execs == 0
+
+
+def test_heat7_graph_does_not_grow_with_the_call(run):
+    """One graph of 48 launches whatever the number of steps, kept for calls of
+    any other number."""
+    first, second, third = run("""
+assert call("heat7", 100003) == 0
+a = log()
+assert call("heat7", 50000) == 0
+b = log()
+assert call("heat7", 195) == 0
+out = [a, b, log()]
+""")
+    graph = "[" + "n" * 48 + "]"
+    assert first.count("[") == 1 and graph in first and first.count("L") < 300
+    assert "[" not in second and second.startswith("R48;") and second.count("L") < 100
+    assert "C" not in first + second  # an even number of launches: nothing to copy back
+    assert "[" not in third

@@ -125,9 +125,10 @@ __global__ void k_ctrl_init(Ctrl *c, double t0, double tend, double cfl) {
 // run time takes about 6 % longer: us a stage, 16x16 / the grid's own shape:
 // 100^3 40.8 / 34.9 (49 and 40 tiles a plane), 190x101x77 50.9 / 48.1 (84 and
 // 78), 33^3 10.1 / 8.6 (9 and 5), 250^3 334 / 348 (256 and 250).
-void small_tile(int nx, int ny, int &tx, int &ty) {
+void small_tile(int nx_, int ny_, int &tx, int &ty) {
+    const long nx = nx_, ny = ny_;  // up to 2^31 - 1 (WENO7): sums of them with a tile's side are 64-bit
     tx = ty = 16;
-    const long t16 = static_cast<long>((nx + 15) / 16) * ((ny + 15) / 16);
+    const long t16 = ((nx + 15) / 16) * ((ny + 15) / 16);
     long best = -1, tiles = 0;
     int bx = 16, by = 16;
     for (int x = kRtSides - 8; x >= 8; x--) {

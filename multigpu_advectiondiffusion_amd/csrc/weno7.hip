@@ -423,8 +423,8 @@ W7Args w7_args(unsigned nx, unsigned ny, unsigned nz, double dx, double dy, doub
     // 25 x 10 for 100 x 100 columns: 40 tiles instead of 49 of 16 x 16, 66.6
     // against 74.6 us a stage at 100^3
     small_tile(g.nx, g.ny, g.tx, g.ty);
-    g.ntx = (g.nx + g.tx - 1) / g.tx;
-    g.nty = (g.ny + g.ty - 1) / g.ty;
+    g.ntx = static_cast<int>((nx + static_cast<unsigned>(g.tx) - 1) / static_cast<unsigned>(g.tx));
+    g.nty = static_cast<int>((ny + static_cast<unsigned>(g.ty) - 1) / static_cast<unsigned>(g.ty));
     const long tiles = static_cast<long>(g.ntx) * g.nty;
     g.kchunk = w7_kchunk(tiles, g.nz, std::max(1, resident_groups(1024)));
     blocks = static_cast<unsigned>(tiles * ((g.nz + g.kchunk - 1) / g.kchunk));

@@ -139,3 +139,19 @@ out = [a, b, log()]
     assert "[" not in second and second.startswith("R48;") and second.count("L") < 100
     assert "C" not in first + second  # an even number of launches: nothing to copy back
     assert "[" not in third
+
+
+@pytest.mark.parametrize("nx,ny", [(n, 1) for n in (2**31 - 1, 2**31 - 34, 2**31 - 35)]
+                         + [(1, n) for n in (2**31 - 1, 2**31 - 32)] + [(7, 2**31 // 7), (3, 2), (100, 100)])
+def test_small_tiles_of_any_accepted_side(nx, ny):
+    """The 256-thread tile of a grid (WENO7 takes sides up to 2^31 - 1): at most
+    256 columns, sides that sum to at most 42, and blocks that cover the grid."""
+    import ctypes
+
+    from multigpu_advectiondiffusion_amd import _capi
+
+    tx, ty = ctypes.c_int(), ctypes.c_int()
+    _capi.lib()._ZN4mgad10small_tileEiiRiS0_(nx, ny, ctypes.byref(tx), ctypes.byref(ty))
+    x, y = tx.value, ty.value
+    assert 1 <= x <= 34 and 1 <= y <= 34 and x * y <= 256 and x + y <= 42
+    assert -(-nx // x) * -(-ny // y) <= -(-nx // 16) * -(-ny // 16)

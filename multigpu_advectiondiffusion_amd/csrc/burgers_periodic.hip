@@ -273,11 +273,22 @@ int square_bands(unsigned nx, unsigned ny, unsigned nz) {
 // warm-up and launch, until 2 to 4 of them share a CU: us a stage, bands of 8
 // against these: 32^3 30 / 9.5 (depth 1), 48^3 21 / 13.3 (2), 64^3 33 / 18
 // (2), 80^3 28 / 24 (2), 96^3 45 / 36 (4), 100^3 51 / 44 (5), 112^3 55 / 49 (6).
+// Columns of more than kMaxBands bands take the next depth, up to 4: us a stage
+// by the general rule and so, 16x16x200 18.4 / 9.4 (2), 27x11x441 25.3 / 15.8
+// (4), 32x32x512 29.5 / 21.4 (4).  From depth 5 on the general rule's 32x16 tiles
+// are faster where they cover the columns well (32x32x640 22.3 / 23.6, 26x30x896
+// 28.0 / 30.9; 16x16x640 17.3 / 15.9).
 int small_kchunk(unsigned nx, unsigned ny, unsigned nz) {
     const long tiles = small_tiles(static_cast<int>(nx), static_cast<int>(ny)), cap = resident_groups(256);
     const int lo = tiles * ((nz + 1) / 2) >= 3 * cap / 16 ? 2 : 1;
-    for (int kc = lo; kc < 8; kc++)
-        if (tiles * ((nz + kc - 1) / kc) <= cap) return static_cast<int>((nz + kc - 1) / kc) <= kMaxBands ? kc : 0;
+    for (int kc = lo; kc < 8; kc++) {
+        const int bands = static_cast<int>((nz + kc - 1) / kc);
+        if (bands > kMaxBands) {
+            if (kc >= 4) return 0;
+            continue;
+        }
+        if (tiles * bands <= cap) return kc;
+    }
     return 0;
 }
 

@@ -28,6 +28,7 @@ std::map<hipStream_t, Capture> captures;
 std::string events;
 int hold_ms = 0;
 int live_execs = 0;
+long last_groups = 0;
 
 struct Config {
     dim3 grid, block;
@@ -71,6 +72,8 @@ int fake_captures_open() {
     std::lock_guard<std::mutex> lock(m);
     return static_cast<int>(captures.size());
 }
+// Workgroups of the last launch.
+long fake_last_groups() { return last_groups; }
 int fake_live_execs() {
     std::lock_guard<std::mutex> lock(m);
     return live_execs;
@@ -87,7 +90,10 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hi
     *stream = config.stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t s) { return work(s, 'L', 'n'); }
+hipError_t hipLaunchKernel(const void *, dim3 g, dim3, void **, size_t, hipStream_t s) {
+    last_groups = 1l * g.x * g.y * g.z;
+    return work(s, 'L', 'n');
+}
 hipError_t hipMemcpyAsync(void *, const void *, size_t, hipMemcpyKind, hipStream_t s) { return work(s, 'C', 'c'); }
 hipError_t hipStreamSynchronize(hipStream_t) { return note('W'); }
 hipError_t hipDeviceSynchronize() { return note('D'); }

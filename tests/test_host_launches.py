@@ -155,3 +155,13 @@ def test_small_tiles_of_any_accepted_side(nx, ny):
     x, y = tx.value, ty.value
     assert 1 <= x <= 34 and 1 <= y <= 34 and x * y <= 256 and x + y <= 42
     assert -(-nx // x) * -(-ny // y) <= -(-nx // 16) * -(-ny // 16)
+
+
+@pytest.mark.parametrize("shape,groups", [((16, 16, 200), 100), ((27, 11, 441), 222), ((32, 32, 512), 512),
+                                          ((16, 16, 64), 64), ((32, 32, 32), 128)])
+def test_thin_periodic_grids_fill_the_device(run, shape, groups):
+    """Columns of more than 128 one-plane bands get the next depth."""
+    assert run(f"""
+assert call("periodic", 1, graph=0, **dict(zip(("nx", "ny", "nz"), {shape}))) == 0
+out = fake.fake_last_groups()
+""") == groups

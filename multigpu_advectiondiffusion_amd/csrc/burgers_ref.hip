@@ -272,35 +272,59 @@ __global__ void k_ref_amax_clear(unsigned long long *amax) {
 
 // What a call needs of u beside its steps, in one pass: max|u| over all nodes
 // into slots 0 and 3, and the three ghost layers, which no stage writes, into
-// the stage buffers w1 and w2.  A wave takes whole rows: rows of the ghost
-// planes and the first and last three of a plane are copied whole, of the
-// others the first and last three nodes.  Bound by the read of u: 8 B a node
-// (1601x986x35: two copies of u and a separate max|u| pass took 490 us a call,
-// this 90).
+// the stage buffers w1 and w2.  A row is ceil(nx / 64) segments of a wave's
+// width, and a wave takes eight consecutive segments at a time, of one row or of
+// several: rows of the ghost planes and the first and last three of a plane are
+// copied whole, of the others the first and last three nodes.  Bound by the
+// read of u, 8 B a node, and on small grids by the atomics on one address, 13
+// ns each: a block leaves them out where the slots already hold as much.
+// us a call's set-up by two copies of u and a separate max|u| pass / by whole
+// rows, one at a time / so: 26x26x300 35 / 52 / 16, 24x1024x1024 215 / 382 / 111,
+// 7x7x4000 33 / 61 / 29, 100^3 74 / 58 / 19, 1601x986x35 439 / 103 / 97.
+constexpr int kPrepSegs = 8;  // segments, and so loads in flight, of a wave
 __global__ __launch_bounds__(256) void k_ref_prepare(const double *__restrict__ u, double *__restrict__ w1,
                                                      double *__restrict__ w2, int nx, int ny, int nz,
                                                      unsigned long long *amax) {
     __shared__ unsigned long long red[4];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const long rows = static_cast<long>(ny) * nz, step = 4l * gridDim.x;
+    const unsigned segs = (static_cast<unsigned>(nx) + 63u) / 64u;
+    const unsigned units = segs * static_cast<unsigned>(ny) * static_cast<unsigned>(nz);  // < 2^31
+    const unsigned groups = (units + kPrepSegs - 1) / kPrepSegs;
     unsigned long long m = 0ull;
-    for (long r = 4l * blockIdx.x + wave; r < rows; r += step) {
-        const int j = static_cast<int>(r % ny), k = static_cast<int>(r / ny);
-        const bool ghost = j < 3 || j >= ny - 3 || k < 3 || k >= nz - 3;
-        const size_t base = static_cast<size_t>(r) * nx;
-        constexpr int U = 8;  // loads in flight
-        for (int i0 = lane; i0 < nx; i0 += 64 * U) {
-            double v[U];
+    for (unsigned g = 4u * blockIdx.x + static_cast<unsigned>(wave); g < groups; g += 4u * gridDim.x) {
+        const unsigned first = g * kPrepSegs, left = units - first;
+        const unsigned r0 = first / segs, s0 = first - r0 * segs, k0 = r0 / static_cast<unsigned>(ny);
+        double v[kPrepSegs];
+        unsigned r = r0, sg = s0;
 #pragma unroll
-            for (int q = 0; q < U; q++) v[q] = u[base + min(i0 + 64 * q, nx - 1)];
+        for (int q = 0; q < kPrepSegs; q++) {
+            const unsigned i = min(sg * 64u + lane, static_cast<unsigned>(nx) - 1u);
+            v[q] = u[static_cast<size_t>(r) * static_cast<unsigned>(nx) + i];
+            if (q + 1u < left && ++sg == segs) {  // past the last segment: the last one again
+                sg = 0;
+                r++;
+            }
+        }
+        r = r0;
+        sg = s0;
+        int j = static_cast<int>(r0 - k0 * static_cast<unsigned>(ny)), k = static_cast<int>(k0);
 #pragma unroll
-            for (int q = 0; q < U; q++) {
-                const unsigned long long b = abs_bits(v[q]);
-                m = b > m ? b : m;
-                const int i = i0 + 64 * q;
-                if (i < nx && (ghost || i < 3 || i >= nx - 3)) {
-                    w1[base + i] = v[q];
-                    w2[base + i] = v[q];
+        for (int q = 0; q < kPrepSegs; q++) {
+            const unsigned long long b = abs_bits(v[q]);
+            m = b > m ? b : m;
+            const int i = static_cast<int>(sg * 64u) + lane;
+            const bool ghost = j < 3 || j >= ny - 3 || k < 3 || k >= nz - 3;
+            if (i < nx && (ghost || i < 3 || i >= nx - 3)) {
+                const size_t o = static_cast<size_t>(r) * static_cast<unsigned>(nx) + static_cast<unsigned>(i);
+                w1[o] = v[q];
+                w2[o] = v[q];
+            }
+            if (q + 1u < left && ++sg == segs) {
+                sg = 0;
+                r++;
+                if (++j == ny) {
+                    j = 0;
+                    k++;
                 }
             }
         }
@@ -311,8 +335,8 @@ __global__ __launch_bounds__(256) void k_ref_prepare(const double *__restrict__ 
     if (threadIdx.x == 0) {
         m = red[0];
         for (int w = 1; w < 4; w++) m = red[w] > m ? red[w] : m;
-        atomicMax(&amax[0], m);
-        atomicMax(&amax[3], m);
+        for (int s : {0, 3})
+            if (m > __hip_atomic_load(&amax[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&amax[s], m);
     }
 }
 
@@ -448,9 +472,11 @@ extern "C" int mgad_burgers_ref_steps(hipStream_t stream, const mgad_scheme *sch
     if (!L.g.amax) return MGAD_ERR_HIP;
     hipLaunchKernelGGL(k_ref_amax_clear, dim3(1), dim3(1), 0, stream, L.g.amax);
     // the stage buffers carry u's ghost layers (never written by any stage)
-    const unsigned rows4 = static_cast<unsigned>((1ull * ny * nz + 3) / 4);
-    hipLaunchKernelGGL(k_ref_prepare, dim3(std::min(rows4, 2048u)), dim3(256), 0, stream, u, w1, w2, (int)nx, (int)ny,
-                       (int)nz, L.g.amax);
+    const unsigned long long units = 1ull * ((nx + 63) / 64) * ny * nz;
+    const unsigned blocks =
+        static_cast<unsigned>(std::min<unsigned long long>((units + 4 * kPrepSegs - 1) / (4 * kPrepSegs), 2048));
+    hipLaunchKernelGGL(k_ref_prepare, dim3(blocks), dim3(256), 0, stream, u, w1, w2, (int)nx, (int)ny, (int)nz,
+                       L.g.amax);
     int st = check_launch();
     if (st) return st;
     const DiffCoef kc = viscous ? diff_coef() : DiffCoef{0.0, 0.0, 0.0};

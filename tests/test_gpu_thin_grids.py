@@ -22,3 +22,28 @@ def test_default_launch_of_thin_grids(hipdev, shape, scheme, kw):
     O.burgers_run(u, (s.dx, s.dy, s.dz), cfl, 0.0, 10.0, nsteps=1, **kw)
     got = s.solution()
     assert np.array_equal(got, u), np.argwhere(got != u)[:5]
+
+
+# the set-up pass takes eight row segments at a time: groups across rows and
+# planes, two and three segments a row, a last group of 1, 3 and 7 segments
+@pytest.mark.parametrize("shape", [(7, 7, 7), (7, 41, 11), (26, 13, 15), (64, 9, 7), (65, 9, 11), (130, 7, 9)])
+def test_reference_set_up_of_narrow_grids(hipdev, shape):
+    nx, ny, nz = shape
+    u = np.random.default_rng(5).uniform(-1.0, 1.0, size=(nz, ny, nx))
+    s = solvers.ReferenceBurgers(shape, 0.1, 0.1, 0.1, scheme="Z1", viscous=False)
+    for w in (s.w1, s.w2):
+        w.upload(np.full((nz, ny, nx), 1e300), s.stream)
+    s.set_initial(u)
+    s.steps(1, 1e-3)
+    for w in (s.w1, s.w2):  # the ghost layers are u's, nothing else was copied
+        g = w.download(s.stream)
+        inner = (slice(3, -3),) * 3
+        assert not np.isin(g[inner], u[inner]).any()
+        g[inner] = u[inner]
+        assert np.array_equal(g, u)
+    Lu, uo = np.zeros_like(u), u.copy()
+    for rk in (1, 2, 3):
+        for axis in range(3):
+            O.adv(axis, u, Lu, 0.1, **O.REFERENCE)
+        O.ssprk_b5(u, uo, Lu, rk, 1e-3)
+    assert np.array_equal(s.solution(), u)

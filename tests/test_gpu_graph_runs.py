@@ -45,3 +45,93 @@ def test_heat7_calls_around_the_graph_length(hipdev, shape, counts):
         b.steps(n, graph=False)
         x = a.solution()
         assert np.isfinite(x).all() and np.array_equal(x, b.solution()), n
+
+
+def test_threads_capture_and_replay_at_the_same_time(hipdev):
+    """Four host threads, each with its own stream and grid, in calls long
+    enough to be captured and replayed, with a remainder: every result equals the
+    same steps launched directly.  The threads issue only work ordered on their
+    own streams, since a device-wide wait would invalidate a capture."""
+    import threading
+
+    sizes = (16, 32, 24, 48)
+    u0s = [solvers.ic_fourier(n, seed=40 + i) for i, n in enumerate(sizes)]
+    direct = []
+    for n, u0 in zip(sizes, u0s):
+        s = solvers.PeriodicBurgers(n)
+        s.set_initial(u0)
+        s.steps(5 * 20, graph=False)
+        direct.append(s.solution())
+    solver = [solvers.PeriodicBurgers(n) for n in sizes]
+    hipdev.synchronize()
+    got, errors = [None] * len(sizes), []
+
+    def work(i):
+        try:
+            solver[i].set_initial(u0s[i])
+            for _ in range(5):
+                solver[i].steps(20, graph=True)
+            got[i] = solver[i].solution()
+        except Exception as e:  # reported below
+            errors.append(repr(e))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(sizes))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=100)
+    assert not errors, errors
+    for x, y in zip(got, direct):
+        assert x is not None and np.array_equal(x, y)
+
+
+def _status(s):
+    st = _capi.BurgersState()
+    rc = _capi.lib().mgad_burgers_read_ctrl(s.stream.handle, s.ctrl.ptr, ctypes.byref(st))
+    _capi.last_error()
+    return rc, st
+
+
+def _time(s):
+    if isinstance(s, solvers.Weno7Burgers):
+        t, _, steps = s.state()
+        return t, steps
+    st = _status(s)[1]
+    return st.t, st.steps
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, 1e200], ids=["nan", "inf", "overflow"])
+def test_a_replayed_graph_stops_at_a_non_finite_value(hipdev, bad):
+    """The graph of a finite run replayed on a field that is not, or stops
+    being so inside the first step: u, t and the step count stay."""
+    n = 32
+    s = solvers.PeriodicBurgers(n)
+    u0 = solvers.ic_fourier(n, seed=8)
+    s.set_initial(u0, tend=10.0)
+    s.steps(20)
+    assert s.state().steps == 20
+    u0[10, 3, 4] = bad
+    s.set_initial(u0, tend=10.0)
+    s.steps(35)
+    rc, st = _status(s)
+    assert rc == _capi.MGAD_ERR_NONFINITE and (st.dt, st.t, st.steps) == (0.0, 0.0, 0)
+    assert np.array_equal(s.solution(), u0, equal_nan=True)
+
+
+@pytest.mark.parametrize("make", [lambda: solvers.PeriodicBurgers((32, 16, 12)),
+                                  lambda: solvers.SlabBurgers((32, 16, 12), 3),
+                                  lambda: solvers.Weno7Burgers((32, 16, 12))],
+                         ids=["periodic", "slab", "weno7"])
+def test_a_run_that_ends_inside_a_graph(hipdev, make):
+    """tend falls inside a replay: the steps after it do nothing."""
+    u0 = 0.5 + 0.4 * np.random.default_rng(9).random((12, 16, 32))
+    a, b = make(), make()
+    b.set_initial(u0)
+    b.steps(25, graph=False)
+    tend = _time(b)[0] - 1e-4
+    for s, calls, graph in ((a, (20, 20, 20), True), (b, (60,), False)):
+        s.set_initial(u0, tend=tend)
+        for n in calls:
+            s.steps(n, graph=graph)
+    assert _time(a) == _time(b) == (tend, 25)
+    assert np.array_equal(a.solution(), b.solution())

@@ -323,12 +323,13 @@ int mgad_burgers_stage(hipStream_t stream, const mgad_scheme *scheme,
                        void *ctrl);
 
 /* nsteps full SSP-RK3 steps: u (in/out) plus two scratch fields w1, w2 of
- * nx*ny*nz doubles.  use_graph != 0 replays a hipGraph of 16 steps, captured by
- * the first call of at least 16 steps with these arguments and kept; the steps
- * left over, the first 64 of the call that captures, and calls of fewer steps
- * are launched directly (the graphs of the other step calls hold about 48
- * launches too).  Asynchronous on stream.  On a stream that the caller is
- * capturing a call with use_graph fails with MGAD_ERR_HIP. */
+ * nx*ny*nz doubles.  use_graph != 0 lets a long run replay a hipGraph of 16
+ * steps: the first 800 steps with the same arguments, in one call or several,
+ * are launched directly, then the graph is captured and kept, and steps beyond
+ * whole graphs are launched directly too (the other step calls do the same with
+ * graphs of about 48 launches, after 50 of them).  Asynchronous on stream.  On a
+ * stream that the caller is capturing a call with use_graph fails with
+ * MGAD_ERR_HIP. */
 int mgad_burgers_steps(hipStream_t stream, const mgad_scheme *scheme,
                        unsigned int nx, unsigned int ny, unsigned int nz,
                        double dx, double dy, double dz, double *u, double *w1,
@@ -432,9 +433,10 @@ int mgad_batch_init(hipStream_t stream, int precision,
                     double tend, double cfl, mgad_batch *out);
 
 /* nsteps SSP-RK3 steps of every problem: three persistent launches per step
- * (each walks the whole work list).  With use_graph all but the first 64 steps
- * are replays of a hipGraph of 16, and the call returns when they have ended
- * (it synchronises the stream); without, it is asynchronous on stream.  Each problem keeps its own dt and LF alpha, and its results are
+ * (each walks the whole work list).  With use_graph a call of more than 800 steps
+ * replays a hipGraph of 16 for the rest, and every call returns when its steps
+ * have ended (it synchronises the stream); without, it is asynchronous on
+ * stream.  Each problem keeps its own dt and LF alpha, and its results are
  * bit-identical to advancing it alone. */
 int mgad_batch_steps(hipStream_t stream, const mgad_batch *batch, int nsteps,
                      int use_graph);
@@ -534,7 +536,7 @@ int mgad_weno7_rhs(hipStream_t stream, unsigned int nx, unsigned int ny,
 
 /* nsteps steps, five stage launches each: u (in/out), scratch fields w1, w2
  * and the carried residual res; steps after tend are no-ops on the device.
- * use_graph replays a hipGraph of 9 steps, as for mgad_burgers_steps. */
+ * use_graph as for mgad_burgers_steps, with graphs of 9 steps after 450. */
 int mgad_weno7_steps(hipStream_t stream, unsigned int nx, unsigned int ny,
                      unsigned int nz, double dx, double dy, double dz,
                      double *u, double *w1, double *w2, double *res,

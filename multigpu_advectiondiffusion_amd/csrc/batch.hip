@@ -378,9 +378,9 @@ int enqueue_serial_step(hipStream_t stream, const mgad_batch &b, const mgad_prob
     return MGAD_OK;
 }
 
-// nsteps times `enqueue` (a step of `launches` launches): with use_graph partly
-// as replays of a graph captured for the call (graphed_steps), and the call
-// returns when the steps have ended.
+// nsteps times `enqueue` (a step of `launches` launches): with use_graph a long
+// call's later steps are replays of a graph captured for it (graphed_steps), and
+// the call returns when the steps have ended.
 template <class F>
 int run_graph(hipStream_t stream, int nsteps, int use_graph, int launches, F &&enqueue) {
     if (!use_graph || stream == nullptr) {
@@ -390,10 +390,10 @@ int run_graph(hipStream_t stream, int nsteps, int use_graph, int launches, F &&e
     }
     int st = refuse_capture(stream);
     if (st) return st;
-    hipGraphExec_t exec = nullptr;
-    st = graphed_steps(stream, nsteps, graph_steps(launches), false, exec, enqueue);
+    KeptGraph g;
+    st = graphed_steps(stream, nsteps, graph_steps(launches), false, g, enqueue);
     const int sst = check_hip(hipStreamSynchronize(stream));
-    if (exec) (void)hipGraphExecDestroy(exec);
+    if (g.exec) (void)hipGraphExecDestroy(g.exec);
     return st ? st : sst;
 }
 

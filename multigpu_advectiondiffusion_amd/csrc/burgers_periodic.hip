@@ -543,8 +543,8 @@ struct GraphKey {
     }
 };
 
-std::map<GraphKey, hipGraphExec_t> &graph_cache() {
-    static std::map<GraphKey, hipGraphExec_t> m;
+std::map<GraphKey, KeptGraph> &graph_cache() {
+    static std::map<GraphKey, KeptGraph> m;
     return m;
 }
 

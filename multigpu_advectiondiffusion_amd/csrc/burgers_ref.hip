@@ -442,8 +442,8 @@ unsigned long long *ref_amax_slots(hipStream_t s) {
 using RefGraphKey = std::tuple<hipStream_t, int, int, double, int, unsigned, unsigned, unsigned, double, double,
                                double, double, double, double, double, double *, double *, double *>;
 
-std::map<RefGraphKey, hipGraphExec_t> &ref_graphs() {
-    static std::map<RefGraphKey, hipGraphExec_t> m;
+std::map<RefGraphKey, KeptGraph> &ref_graphs() {
+    static std::map<RefGraphKey, KeptGraph> m;
     return m;
 }
 

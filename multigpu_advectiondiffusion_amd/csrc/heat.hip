@@ -952,7 +952,7 @@ extern "C" int mgad_heat7_fe_steps(hipStream_t stream, unsigned int nx, unsigned
     if (graphs > 0 && left > 0 && left < 2 * t) graphs--;
     int st = MGAD_OK;
     if (graphs > 0) {
-        static std::map<HeatKey, hipGraphExec_t> cache;
+        static std::map<HeatKey, KeptGraph> cache;
         const HeatKey key{stream, nx, ny, nz, kx, ky, kz, dt, u, w};
         st = replay_steps(cache, 16, key, stream, graphs * per, per, [&] {
             const int r = enqueue_heat7(stream, nx, ny, nz, kx, ky, kz, dt, u, w, t);
@@ -992,7 +992,7 @@ extern "C" int mgad_heat13_rk3_steps(hipStream_t stream, unsigned int nx, unsign
     } else {
         using Key = std::tuple<hipStream_t, unsigned, unsigned, unsigned, double, double, double, double, double *,
                                double *>;
-        static std::map<Key, hipGraphExec_t> cache;
+        static std::map<Key, KeptGraph> cache;
         const Key key{stream, nx, ny, nz, c.kx, c.ky, c.kz, dt, u, w1};
         st = replay_steps(cache, 16, key, stream, pairs, graph_steps(2), pair);
     }

@@ -241,7 +241,7 @@ extern "C" int mgad_burgers_slab_steps(hipStream_t stream, const mgad_scheme *sc
     const LaunchCfg cfg = launch_cfg(MGAD_F64, *scheme, nx, ny, nzs * nslab);
     using Key = std::tuple<hipStream_t, int, int, double, unsigned, unsigned, unsigned, unsigned, double, double,
                            double, double *, double *, double *, void *, int, int>;
-    static std::map<Key, hipGraphExec_t> cache;
+    static std::map<Key, KeptGraph> cache;
     const Key key{stream, scheme->weno, scheme->p, scheme->eps, nx, ny, nzs, nslab, dx, dy, dz, u, w1, w2, ctrl,
                   cfg.tile, cfg.kchunk};
     return replay_steps(cache, 16, key, stream, nsteps, graph_steps(3), [&] {

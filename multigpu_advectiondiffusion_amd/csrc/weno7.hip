@@ -505,7 +505,7 @@ extern "C" int mgad_weno7_steps(hipStream_t stream, unsigned int nx, unsigned in
     if (const int st = refuse_capture(stream)) return st;
     using Key = std::tuple<hipStream_t, unsigned, unsigned, unsigned, double, double, double, double *, double *,
                            double *, double *, void *>;
-    static std::map<Key, hipGraphExec_t> cache;
+    static std::map<Key, KeptGraph> cache;
     const Key key{stream, nx, ny, nz, dx, dy, dz, u, w1, w2, res, ctrl};
     return replay_steps(cache, 16, key, stream, nsteps, graph_steps(5), [&] {
         return enqueue_w7_step(stream, nx, ny, nz, dx, dy, dz, u, w1, w2, res, c);

@@ -31,8 +31,12 @@ def run(tmp_path_factory):
     return go
 
 
-# a call long enough to be captured
-LONG = {"periodic": 20, "slab": 20, "reference": 20, "weno7": 20, "heat13": 101, "heat7": 203}
+# launches a step, steps a graph, launches before a call's first step
+SHAPE = {"periodic": (3, 16, 0), "slab": (3, 16, 0), "reference": (3, 16, 2), "weno7": (5, 9, 0),
+         "heat13": (1, 48, 0)}
+DIRECT = 50  # graphs' worth of steps launched before a capture
+# steps of a call long enough to be captured (heat7: 4 steps a launch)
+LONG = {**{k: (DIRECT + 1) * per + 4 for k, (_, per, _) in SHAPE.items()}, "heat7": (DIRECT + 1) * 48 * 4 + 11}
 
 
 @pytest.mark.parametrize("kind", LONG)
@@ -84,43 +88,66 @@ out = [under_capture(2, 1), under_capture(250, 1), under_capture(2, 0)]
     assert out[2][0] == 0 and "n" in out[2][1]
 
 
-# launches a step, steps a graph, launches before a call's first step
-SHAPE = {"periodic": (3, 16, 0), "slab": (3, 16, 0), "reference": (3, 16, 2), "weno7": (5, 9, 0),
-         "heat13": (1, 48, 0)}
-
-
 @pytest.mark.parametrize("kind", SHAPE)
-def test_first_long_call_launches_before_it_captures(run, kind):
-    """The device has work when the host captures; later calls replay, and so
-    does the first one once four graphs' worth of steps has been launched."""
+def test_runs_are_captured_after_fifty_graphs_of_direct_steps(run, kind):
+    """Short runs never capture; a longer one does while the device still has
+    work, in whichever call it gets there, and replays from then on."""
     per_step, per, pre = SHAPE[kind]
-    n, many = per + 4, 6 * per + 4
-    first, second, other = run(f"""
-assert call({kind!r}, {n}) == 0
-a = log()
-assert call({kind!r}, {n}) == 0
-b = log()
-assert call({kind!r}, {many}, u=0x800000) == 0
-out = [a, b, log()]
+    lead = DIRECT * per
+    calls = [lead - 2, per + 6, per + 4, 1]
+    *log, other, short = run(f"""
+out = []
+for n in {calls}:
+    assert call({kind!r}, n) == 0
+    out.append(log())
+assert call({kind!r}, {lead + 2 * per + 4}, u=0x800000) == 0
+out.append(log())
+for _ in range({DIRECT + 2}):
+    assert call({kind!r}, {per - 1}, u=0x900000) == 0
+out.append(log())
 """)
-    nodes = per * per_step
-    graph, replay, rest = "[" + "n" * nodes + "]", f"R{nodes};", "L" * (4 * per_step)
-    assert first == "L" * (pre + n * per_step) + graph
-    assert second == "L" * pre + replay + rest
-    assert other == "L" * (pre + 4 * nodes) + graph + 2 * replay + rest
+    def direct(steps):
+        return "L" * (steps * per_step)
+
+    head, nodes = "L" * pre, per * per_step
+    graph, replay = "[" + "n" * nodes + "]", f"R{nodes};"
+    assert log[0] == head + direct(lead - 2)
+    assert log[1] == head + direct(2) + graph + replay + direct(4)
+    assert log[2] == head + replay + direct(4)
+    assert log[3].count("L") == pre + per_step and "R" not in log[3]
+    assert other == head + direct(lead) + graph + 2 * replay + direct(4)
+    assert "[" not in short
 
 
 @pytest.mark.parametrize("kind,per_step", [("batch", 3), ("serial", 6)])
 def test_batch_call_captures_only_what_it_replays_itself(run, kind, per_step):
+    lead = DIRECT * 48
     short, long, execs = run(f"""
-assert call({kind!r}, {192 // per_step}) == 0
+assert call({kind!r}, {lead // per_step}) == 0
 a = log()
-assert call({kind!r}, {96 * 4 // per_step + 1}) == 0
+assert call({kind!r}, {(lead + 192) // per_step + 1}) == 0
 out = [a, log(), fake.fake_live_execs()]
 """)
-    assert short == "L" * 192 + "W"
-    assert long == "L" * 192 + "[" + "n" * 48 + "]" + 4 * "R48;" + "L" * per_step + "W"
+    assert short == "L" * lead + "W"
+    assert long == "L" * lead + "[" + "n" * 48 + "]" + 4 * "R48;" + "L" * per_step + "W"
     assert execs == 0
+
+
+def test_full_cache_makes_room(run):
+    """Keys without a graph go without a wait; graphs are destroyed after one."""
+    one, kept, full, execs = run(f"""
+for i in range(100):
+    assert call("periodic", 20, u=0x1000000 + 0x1000 * i) == 0
+a = log()
+for i in range(33):
+    assert call("periodic", {LONG["periodic"]}, u=0x2000000 + 0x1000 * i) == 0
+b = log()
+assert call("periodic", 20) == 0
+out = [a, b, log(), fake.fake_live_execs()]
+""")
+    assert set(one) == {"L"}
+    assert kept.count("[") == 33 and "D" not in kept
+    assert full == "D" + "L" * 60 and execs == 0
 
 
 def test_heat7_graph_does_not_grow_with_the_call(run):
@@ -135,8 +162,8 @@ assert call("heat7", 195) == 0
 out = [a, b, log()]
 """)
     graph = "[" + "n" * 48 + "]"
-    assert first.count("[") == 1 and graph in first and first.count("L") < 300
-    assert "[" not in second and second.startswith("R48;") and second.count("L") < 100
+    assert first.count("[") == 1 and graph in first and first.count("L") < (DIRECT + 2) * 48
+    assert "[" not in second and second.startswith("R48;") and second.count("L") < 2 * 48
     assert "C" not in first + second  # an even number of launches: nothing to copy back
     assert "[" not in third
 

@@ -72,13 +72,13 @@ def read_valu(workload: str):
 
 def run_to_half(scheme: str, n: int = 256, seed: int = 3) -> dict:
     """The 256^3 periodic run from the seeded Fourier field to t = 0.5 (past
-    shock formation), one hipGraph replay per step; steps after t = 0.5 are
-    no-ops on the device, so the loop asks for a few more than needed."""
+    shock formation), 64 steps a call; steps after t = 0.5 are no-ops on the
+    device, so the loop asks for a few more than needed."""
     from multigpu_advectiondiffusion_amd import hip, solvers
 
     s = solvers.PeriodicBurgers(n, scheme=scheme, cfl=0.4)
     s.set_initial(solvers.ic_fourier(n, seed=seed), t0=0.0, tend=0.5)
-    s.steps(1)  # capture
+    s.steps(1)
     s.set_initial(solvers.ic_fourier(n, seed=seed), t0=0.0, tend=0.5)
     e0, e1 = hip.Event(), hip.Event()
     hip.synchronize()

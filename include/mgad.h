@@ -366,7 +366,8 @@ int mgad_burgers_steps_p(int precision, hipStream_t stream,
  * tiles may cover at most 7 % more columns than the grid), 256-thread tiles
  * (16x16, or a shape of the grid's own that needs fewer of them) in bands of
  * fewer than 8 planes where deeper ones would leave the device short of
- * workgroups, and otherwise 32x16 or 256-thread tiles, whichever covers the
+ * workgroups (at most 128 bands, of up to 4 planes where shallower ones would be
+ * more), and otherwise 32x16 or 256-thread tiles, whichever covers the
  * grid with less waste; tile 16 means the 256-thread tiles; kchunk > 0 makes
  * the bands kchunk planes deep (4..128 and nz are tried), MGAD_BANDS_SHRINK
  * makes them shrink towards the top of the grid.  Overwrites w1 and ctrl: call mgad_burgers_init[_p]
@@ -633,7 +634,8 @@ int mgad_check_division(hipStream_t stream, int mode, const double *a,
  * main.cpp:108-121): the same u as nsteps times {uo <- u; for rk = 1..3:
  * Call_Lu3d, Call_RK3d(rk)} with the CopyToConstantMemory coefficients, bit
  * for bit, one launch per step.  Interior nodes 2..n-3 are updated, the two
- * ghost layers kept; w1, w2 are scratch fields of the same size.
+ * ghost layers kept; w1 is a scratch field of the same size.  w2 is not touched,
+ * but has to be a third pointer that is neither null nor u or w1.
  * Requires n >= 5 per axis, nx*ny*nz < 2^31 and nx*ny < 2^29. */
 int mgad_heat13_rk3_steps(hipStream_t stream, unsigned int nx, unsigned int ny,
                           unsigned int nz, double dt, double *u, double *w1,

@@ -410,8 +410,10 @@ template int burgers_init_t<float>(hipStream_t, unsigned, unsigned, unsigned, co
 // ---------------------------------------------------------------------------
 // Launch configuration: environment override (MGAD_TILE, MGAD_KCHUNK), then
 // the per-shape table that mgad_burgers_autotune / mgad_burgers_set_launch
-// fill, then the default (32-wide tiles when they divide nx, kchunk from
-// default_kchunk).  Every configuration computes bit-identical results.
+// fill, then the default: one round of 32x32 tiles (square_bands), shallow
+// bands of 256-thread tiles on small grids (small_kchunk), or else the tiles of
+// pick() in bands of default_kchunk or default_kchunk256 planes.  Every
+// configuration computes bit-identical results.
 // ---------------------------------------------------------------------------
 namespace {
 

@@ -95,7 +95,8 @@ __device__ __forceinline__ unsigned long long ref_stage_tile(const double *__res
     // otherwise keep six more doubles in registers), sp/sn[R(q)] the 13/12
     // terms centred on plane k-1+q.  The march is unrolled by 7, so every slot
     // is a constant and no register moves shift the rings (1601x986x35: 6009
-    // to 5813 us a call of 2 steps, spills 8 to 0; 512^3 unchanged).
+    // to 5813 us a call of 2 steps, spills 8 to 0; 512^3, on 32x32 tiles, unchanged:
+    // they still spill 7 with WENO-Z and 3 with JS, in the viscous kernels).
     double qp[7], qm[7], uq[7], sp[7], sn[7];
 #pragma unroll
     for (int q = 0; q < 6; q++) {

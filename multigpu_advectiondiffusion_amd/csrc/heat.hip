@@ -327,7 +327,7 @@ __device__ __forceinline__ StepTile step_tile(unsigned tile, int nx, int ny, int
 // and stage, on 1.8 times the nodes (6 halo nodes a side of 64 x 36), less the
 // waves and planes that a stage does not need, which skip it (1.5 times is
 // left).  One launch per stage was bound by memory: 161 us a step at
-// 201x199x200 and 2021 at 512^3 (4.3 TB/s), now 73 and 915 us (147 Gpts/s).
+// 201x199x200 and 2021 at 512^3 (4.3 TB/s), now 66 and 920 us (146 Gpts/s).
 template <int W, int R>
 __global__ __launch_bounds__(64 * W) void k_heat13_step(const double *__restrict__ u, double *__restrict__ v, int nx,
                                                         int ny, int nz, int ntx, int nty, int kchunk, double kx,
@@ -483,7 +483,7 @@ __global__ __launch_bounds__(64 * W) void k_heat13_step(const double *__restrict
 // is that of k_heat13_step: at iteration k step l = 1..T is computed on plane
 // k - l, whose z neighbours are the last two planes of step l - 1 in registers
 // and the one just computed.  At 512^3 one step a launch is bound by memory
-// (5.6 TB/s, 384 us a step); with 4 (172 us) the FP64 issue time is about 90
+// (5.6 TB/s, 388 us a step); with 4 (174 us) the FP64 issue time is about 90
 // us (16 slots a node and step on 64/(64-2T) * E/(E-2T) times the nodes) and
 // the memory time 100 us, and the barrier of each plane keeps them from
 // overlapping fully.  At 64^3 it is the launch and first-load latency, paid
@@ -841,10 +841,11 @@ int enqueue_heat7(hipStream_t s, unsigned nx, unsigned ny, unsigned nz, double k
 }
 
 // Most steps a launch takes: 4, or 5 where the tall tile is taken.  A
-// fifth step costs the tall tile little (us a step at 512^3 with 2, 3, 4, 5
-// steps a launch: 304, 188, 172, 185; with 1: 384) and saves launches that
-// would only make their number even; the low tile loses more of its rows to
-// the halo (64^3: 2.59, 2.47, 2.43, 2.88; with 1: 3.23).
+// fifth step costs the tall tile next to nothing (us a step with 1, 2, 3, 4, 5
+// steps a launch: 512^3 388, 301, 185, 174, 177; 201x199x200 26.4, 16.9, 13.0,
+// 12.4, 12.3) and saves launches that would only make their number even; the
+// low tile loses more of its rows to the halo (64^3 by the march: 3.23, 2.59,
+// 2.47, 2.43, 2.88).
 int heat7_most_steps(unsigned nx, unsigned ny, unsigned nz) {
     bool tall;
     heat7_steps_grid(nx, ny, nz, 4, tall);

@@ -12,11 +12,10 @@
 batched: 64 independent periodic WENO5-Z (p=2, eps=1e-40) FP64 problems with
     edge lengths drawn seeded-uniformly from {32,48,64,96,128} (SplitMix64 seed
     4), each with its own Fourier initial field (seed 4+i) and its own dt from
-    CFL 0.4, advanced `steps` steps (a) in one persistent launch per RK stage
-    under a hipGraph-captured step, (b) problem by problem with the
-    single-problem kernel, each size autotuned and each step a replayed
-    hipGraph, and (c) problem by problem with eager launches of the default
-    launch shape.  Reports the throughputs (points * steps / s) and the
+    CFL 0.4, advanced `steps` steps (a) in one persistent launch per RK stage,
+    (b) problem by problem with the single-problem kernel, each size autotuned
+    (both allowed step graphs, which replay steps of long calls only), and (c)
+    problem by problem with eager launches of the default launch shape.  Reports the throughputs (points * steps / s) and the
     ratios of (a) to (b) and to (c).
 fp32: the same Burgers setup with WENO5-Z at n^3, run to t = 0.5 once in FP64
     and once with FP32 storage (FP64 split fluxes, smoothness indicators and
@@ -110,7 +109,7 @@ def batched(steps: int = 200, nprob: int = 64, scheme: str = "Z2") -> dict:
 
     def timed(fn):
         b.set_initial(u0s, tend=float("inf"), kchunk=0)
-        fn(2)  # builds the graph once
+        fn(2)
         warm(lambda: fn(4))
         b.set_initial(u0s, tend=float("inf"), kchunk=b.batch.kchunk)
         hip.synchronize()
@@ -310,7 +309,7 @@ def reference_cases(cases=REFERENCE_CASES, dropin_steps: int = 3) -> dict:
         u0 = fileio.init3d_burgers(3, (nx, ny, nz), dx, dy, dz)
         s = solvers.ReferenceBurgers((nx, ny, nz), dx, dy, dz, scheme="Z1", viscous=True)
         s.set_initial(u0)
-        s.steps(1, dt)  # graph capture
+        s.steps(1, dt)
         warm(lambda: s.steps(2, dt))
         s.set_initial(u0)
         hip.synchronize()
@@ -382,7 +381,7 @@ def heat_cases(dropin_steps: int = 5) -> dict:
     for n, steps in ((64, 100), (512, 20)):
         h = solvers.Heat7(n)
         h.set_initial(solvers.ic_gauss_noise(n, seed=1))
-        h.steps(steps)  # graph capture
+        h.steps(steps)
         warm(lambda: h.steps(steps))
         t = timed(h.stream, lambda: h.steps(steps))
         gbs = 16.0 * n ** 3 * steps / t / 1e9
@@ -397,7 +396,7 @@ def heat_cases(dropin_steps: int = 5) -> dict:
     u0 = fileio.init3d_heat(3, (nx, ny, nz), dx, dy, dz)
     h = solvers.ReferenceHeat((nx, ny, nz))
     h.set_initial(u0)
-    h.steps(1, dt)  # graph capture
+    h.steps(1, dt)
     warm(lambda: h.steps(20, dt))
     h.set_initial(u0)
     t = timed(h.stream, lambda: h.steps(iters, dt))
@@ -416,12 +415,11 @@ def heat_cases(dropin_steps: int = 5) -> dict:
                  "fused_vs_dropin": (npts * iters / t) / (npts * dropin_steps / td)})
     out["reference_heat13_rk3"] = case
     del h, du, duo, dLu
-    # the same fused step on a 512^3 grid (bandwidth once launches are long;
-    # the timed call includes its two initial field copies, ~2 %)
+    # the same fused step on a 512^3 grid
     n, steps = 512, 20
     h = solvers.ReferenceHeat((n, n, n))
     h.set_initial(solvers.ic_gauss_noise(n, seed=1))
-    h.steps(1, 1e-6)  # graph capture
+    h.steps(1, 1e-6)
     warm(lambda: h.steps(2, 1e-6))
     t = timed(h.stream, lambda: h.steps(steps, 1e-6))
     out["heat13_rk3_512"] = {"steps": steps, "gpts": n ** 3 * steps / t / 1e9,
@@ -517,8 +515,8 @@ def adjoint_trace(n: int = 128, steps: int = 100, copy_calib: bool = False) -> d
 
 def batched_trace(steps: int = 20, nprob: int = 64, scheme: str = "Z2") -> dict:
     """The batched path alone on the batched study's 64 problems: the
-    autotuner's timing runs, then `steps` hipGraph-replayed steps with the
-    work list it picked (the workload of the batched kernel trace)."""
+    autotuner's timing runs, then `steps` steps with the work list it picked
+    (the workload of the batched kernel trace)."""
     sizes = batch_sizes(nprob)
     u0s = [solvers.ic_fourier(n, seed=4 + i) for i, n in enumerate(sizes)]
     b = solvers.BurgersBatch(sizes, scheme=scheme)

@@ -281,7 +281,8 @@ __global__ void k_ref_amax_clear(unsigned long long *amax) {
 // ns each: a block leaves them out where the slots already hold as much.
 // us a call's set-up by two copies of u and a separate max|u| pass / by whole
 // rows, one at a time / so: 26x26x300 35 / 52 / 16, 24x1024x1024 215 / 382 / 111,
-// 7x7x4000 33 / 61 / 29, 100^3 74 / 58 / 19, 1601x986x35 439 / 103 / 97.
+// 7x7x4000 33 / 61 / 29, 100^3 74 / 58 / 19, 1601x986x35 439 / 103 / 97 (twice a
+// call of one step less a call of two; the pass itself takes 120 us there).
 constexpr int kPrepSegs = 8;  // segments, and so loads in flight, of a wave
 __global__ __launch_bounds__(256) void k_ref_prepare(const double *__restrict__ u, double *__restrict__ w1,
                                                      double *__restrict__ w2, int nx, int ny, int nz,
